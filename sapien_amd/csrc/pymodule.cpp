@@ -291,14 +291,17 @@ std::unique_ptr<DLIn> take(const py::object &t, uint8_t code, const std::vector<
 
 // A float32 GPU tensor whose last dimension is contiguous and whose other
 // dimensions may be strided (padded buffers, slices of them): shape entries
-// < 0 are free; returns the element strides.
+// < 0 are free; returns the element strides. A dimension of several entries with
+// stride 0 (an expanded tensor) is refused: to the C ABI a stride of 0 means
+// contiguous rows, which such a tensor does not have.
 std::unique_ptr<DLIn> take_strided(const py::object &t, const std::vector<int64_t> &shape, int device) {
   Torch &T = Torch::get();
   if (shape.size() <= 8 && T.on_device(t, T.f32, device) && !T.flag(t, T.n_requires_grad)) {
     int64_t dims[8], steps[8];
     const int n = (int)shape.size();
     bool good = T.sizes(T.attr(t, T.n_shape), dims, 8) == n && T.sizes(T.call(t, T.n_stride), steps, 8) == n;
-    for (int i = 0; good && i < n; ++i) good = (shape[i] < 0 || dims[i] == shape[i]) && steps[i] >= 0;
+    for (int i = 0; good && i < n; ++i)
+      good = (shape[i] < 0 || dims[i] == shape[i]) && (steps[i] > 0 || (steps[i] == 0 && dims[i] <= 1));
     if (good && (n == 0 || dims[n - 1] <= 1 || steps[n - 1] == 1)) {
       auto in = std::make_unique<DLIn>();
       in->strides.assign(steps, steps + n);
@@ -329,8 +332,11 @@ std::unique_ptr<DLIn> take_strided(const py::object &t, const std::vector<int64_
   }
   if (d.ndim > 0 && d.shape[d.ndim - 1] > 1 && in->strides[d.ndim - 1] != 1)
     throw py::value_error("the last dimension of a strided buffer must be contiguous");
-  for (int i = 0; i < d.ndim; ++i)
+  for (int i = 0; i < d.ndim; ++i) {
     if (in->strides[i] < 0) throw py::value_error("negative strides are not supported");
+    if (in->strides[i] == 0 && d.shape[i] > 1)
+      throw py::value_error("expanded tensors (stride 0) are not supported: the rows must be in memory");
+  }
   in->ptr = static_cast<char *>(d.data) + d.byte_offset;
   return in;
 }
@@ -597,16 +603,24 @@ class PyModel {
     StreamScope scope_(stream, info().device);
     sapamd_info i = info();
     Torch &T = Torch::get();
+    // rows of an expanded tensor are copied out: the kernel reads rows in memory
+    auto in_memory = [&](py::object x) {
+      int64_t dims[2], steps[2];
+      if (T.sizes(T.attr(x, T.n_shape), dims, 2) == 2 && T.sizes(T.call(x, T.n_stride), steps, 2) == 2 &&
+          dims[0] > 1 && steps[0] == 0 && (dims[1] <= 1 || steps[1] == 1))
+        return py::object(x.attr("contiguous")());
+      return x;
+    };
     auto as_gpu = [&](py::object x) {
       int64_t dims[2];
       if (T.on_device(x, T.f32, i.device) && T.sizes(T.attr(x, T.n_shape), dims, 2) == 2)
-        return T.flag(x, T.n_requires_grad) ? py::object(x.attr("detach")()) : x;
+        return in_memory(T.flag(x, T.n_requires_grad) ? py::object(x.attr("detach")()) : x);
       py::module_ torch = py::module_::import("torch");
       if (!py::isinstance(x, torch.attr("Tensor"))) x = torch.attr("as_tensor")(x);
       x = x.attr("detach")().attr("to")(py::arg("device") = py::reinterpret_borrow<py::object>(T.device(i.device)),
                                         py::arg("dtype") = torch.attr("float32"));
       if (x.attr("dim")().cast<int>() == 1) x = x.attr("unsqueeze")(0);
-      return x;
+      return in_memory(x);
     };
     q = as_gpu(q);
     auto vq = take_strided(q, {-1, i.nv}, i.device);

@@ -98,3 +98,33 @@ def test_streams(arm):
     side.synchronize()
     assert torch.equal(got, want) and torch.equal(raw, want)
     assert np.isfinite(want.cpu().numpy()).all()
+
+
+def test_expanded_rows(arm):
+    """One row standing for all of them (stride 0): copied out where inputs are
+    converted, refused where buffers are used in place."""
+    m, (q, qd, _, _) = arm
+    B, n = q.shape
+    eq, eqd = q[:1].expand(B, n), qd[0].expand(B, n)
+    rows = [x.contiguous() for x in (eq, eqd)]
+    for f in (lambda x: x, lambda x: x.clone()[:1].expand(B, n).requires_grad_(True), torch.Tensor.double,
+              lambda x: x.as_subclass(_Sub)):
+        assert torch.equal(m.compute_passive_force_batched(f(eq), f(eqd)), m.compute_passive_force_batched(*rows))
+        assert torch.equal(m.compute_forward_kinematics_batched(f(eq)), m.compute_forward_kinematics_batched(rows[0]))
+    poses, tau = torch.empty(B, m.nlinks, 7, device="cuda"), torch.empty(B, n, device="cuda")
+    body = torch.zeros(B, m.nlinks, 13, device="cuda")
+    for bad in (eq, eq.as_subclass(_Sub)):
+        for call in (lambda: m.compute_fk_jacobian_rnea_into(bad, poses=poses),
+                     lambda: m.compute_fk_jacobian_rnea_into(q, qvel=bad, qacc=q, qf=tau),
+                     lambda: m.compute_fk_jacobian_rnea_into(q, qvel=q, qacc=q, qf=bad),
+                     lambda: m.compute_fk_jacobian_rnea_into(q, poses=poses[:1].expand_as(poses)),
+                     lambda: m.compute_fk_jacobian_rnea_into(q, poses=poses[:, :1].expand_as(poses)),
+                     lambda: m.compute_link_state_into(bad, body=body),
+                     lambda: m.compute_link_state_into(q, qvel=bad, body=body),
+                     lambda: m.compute_link_state_into(q, body=body[:1].expand_as(body)),
+                     lambda: m.compute_passive_force_batched(q, qd, out=bad)):
+            with pytest.raises(ValueError, match="expanded"):
+                call()
+    one = q[:1].as_strided((1, n), (0, 1))  # the stride of a single row says nothing
+    m.compute_fk_jacobian_rnea_into(one, qvel=one, qacc=one, qf=tau[:1])
+    assert torch.equal(tau[:1], m.compute_inverse_dynamics_batched(q[:1], q[:1], q[:1]))
