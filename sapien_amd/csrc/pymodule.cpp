@@ -135,13 +135,26 @@ struct Torch {
   py::handle n_dtype, n_layout, n_is_cuda, n_get_device, n_shape, n_contiguous, n_data_ptr, n_requires_grad, n_stride;
   std::vector<py::handle> devices;  // torch.device("cuda", i)
 
+  // A plain pointer read and written under the GIL, not a static with an
+  // initializer: importing torch lets other threads run, and one that waited at
+  // the initializer's guard would hold the GIL that the import needs. A thread
+  // that gets here meanwhile builds one of its own; the first one stays.
   static Torch &get() {
-    static Torch *t = new Torch;
-    return *t;
+    static Torch *kept = nullptr;
+    if (!kept) {
+      Torch *made = new Torch;
+      if (!kept) kept = made;
+      else delete made;
+    }
+    return *kept;
   }
   py::handle device(int i) {
     if (i < 0) device_type("cuda", i);  // no GPU: torch raises
-    while ((int)devices.size() <= i) devices.push_back(device_type("cuda", (int)devices.size()).release());
+    while ((int)devices.size() <= i) {
+      const size_t n = devices.size();
+      py::object d = device_type("cuda", (int)n);
+      if (devices.size() == n) devices.push_back(d.release());  // no other thread was quicker
+    }
     return devices[i];
   }
   // A tensor whose attributes can be read at face value: torch.Tensor itself or

@@ -2,6 +2,10 @@
 a DLPack capsule that claims this model's (absent) GPU gets as far as torch's
 stream of that GPU, unless the binding refuses it first."""
 import ctypes
+import os
+import subprocess
+import sys
+import textwrap
 
 import pytest
 
@@ -74,3 +78,40 @@ def test_expanded_tensors_are_refused_in_place(arm):
     one = _on_device(torch.zeros(1, nv).as_strided((1, nv), (0, 1)))
     with pytest.raises(RuntimeError, match=TAKEN):
         into(one, qvel=one, qacc=one, qf=one)
+
+
+def test_first_calls_from_two_threads():
+    """The first batched calls of a process, from two threads at once, on numpy
+    arrays and with torch not imported yet: both come back (here with torch's
+    error for want of a GPU)."""
+    script = textwrap.dedent("""
+        import sys, threading
+        import numpy as np
+        import sapien_amd as sa
+        from sapien_amd import synthetic as S
+        assert "torch" not in sys.modules
+        rob, gate, out = S.chain7(), threading.Barrier(2), [None, None]
+        models = []
+        for _ in out:
+            m = sa.PinocchioModel(rob.urdf, [0.0, 0.0, -9.81])
+            m.set_joint_order(rob.joint_names)
+            m.set_link_order(rob.link_names)
+            models.append(m)
+
+        def call(i):
+            gate.wait()
+            try:
+                out[i] = "poses", models[i].compute_forward_kinematics_batched(np.zeros((2, rob.nv))).shape
+            except RuntimeError as e:
+                out[i] = "error", str(e)
+
+        threads = [threading.Thread(target=call, args=(i,)) for i in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert out[0] and out[0] == out[1], out
+        """)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    env = dict(os.environ, PYTHONPATH=root, HIP_VISIBLE_DEVICES="")
+    subprocess.run([sys.executable, "-c", script], env=env, check=True, timeout=120)
