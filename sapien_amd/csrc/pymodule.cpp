@@ -191,9 +191,11 @@ struct Torch {
     if (!p && PyErr_Occurred()) throw py::error_already_set();
     return p;
   }
-  // The shape of a tensor or of anything torch.as_tensor takes.
+  // The shape of a tensor, of anything else that DLPack can hand over, or of
+  // anything torch.as_tensor takes.
   std::vector<int64_t> shape(const py::object &x) const {
-    const py::object t = plain(x) ? x : py::module_::import("torch").attr("as_tensor")(x);
+    const bool own = plain(x) || py::hasattr(x, "__dlpack__");
+    const py::object t = own ? x : py::module_::import("torch").attr("as_tensor")(x);
     return attr(t, n_shape).cast<std::vector<int64_t>>();
   }
   // Sizes of a tuple of ints (a shape or strides).

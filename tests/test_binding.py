@@ -53,6 +53,29 @@ def arm():
     return m, rob.nv
 
 
+class _Foreign:
+    """No torch tensor: a shape and a DLPack capsule."""
+
+    def __init__(self, x):
+        self.tensor, self.shape = _on_device(x), tuple(x.shape)
+
+    def __dlpack__(self, **kw):
+        return self.tensor.__dlpack__()
+
+
+@needs_no_gpu
+def test_dlpack_objects_that_torch_does_not_know(arm):
+    """The in-place methods take their buffers through DLPack alone."""
+    (m, nv), B, L = arm, 3, arm[0].nlinks
+    q, poses, body = (_Foreign(torch.zeros(s)) for s in ((B, nv), (B, L, 7), (B, L, 13)))
+    with pytest.raises(RuntimeError, match=TAKEN):
+        m.compute_fk_jacobian_rnea_into(q, qvel=q, qacc=q, poses=poses, qf=q)
+    with pytest.raises(RuntimeError, match=TAKEN):
+        m.compute_link_state_into(q, qvel=q, body=body)
+    with pytest.raises(ValueError, match=">= nlinks"):
+        m.compute_fk_jacobian_rnea_into(q, poses=_Foreign(torch.zeros(B, L - 1, 7)))
+
+
 @needs_no_gpu
 def test_expanded_tensors_are_refused_in_place(arm):
     """A row, environment or link stride of 0 over several entries: the C ABI
