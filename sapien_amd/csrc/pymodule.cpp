@@ -826,7 +826,8 @@ class PyModel {
           t->attr("dtype").ptr() != b.T.f32.ptr() || !t->attr("is_cuda").cast<bool>())
         throw std::runtime_error("rollout_step_ needs contiguous float32 GPU tensors");
     }
-    auto vq = take(q, dlabi::kFloat, {b.B, b.n}, b.device), vqd = take(qd, dlabi::kFloat, {b.B, b.n}, b.device),
+    // q also as one row without its batch dimension (Batch has checked its size)
+    auto vq = take(q, dlabi::kFloat, b.T.shape(q), b.device), vqd = take(qd, dlabi::kFloat, {b.B, b.n}, b.device),
          vt = take(tau_t, dlabi::kFloat, {b.B, b.n}, b.device);
     check(sapamd_rollout_step(m_, b.B, (float)dt, f(vq), f(vqd), f(vt), b.n, b.stream(stream)));
   }

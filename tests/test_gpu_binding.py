@@ -128,3 +128,15 @@ def test_expanded_rows(arm):
     one = q[:1].as_strided((1, n), (0, 1))  # the stride of a single row says nothing
     m.compute_fk_jacobian_rnea_into(one, qvel=one, qacc=one, qf=tau[:1])
     assert torch.equal(tau[:1], m.compute_inverse_dynamics_batched(q[:1], q[:1], q[:1]))
+
+
+def test_rollout_step_on_one_row(arm):
+    """One environment's configuration without its batch dimension, updated in place."""
+    m, (q, qd, _, tau) = arm
+    want = q[:1].clone(), qd[:1].clone()
+    m.rollout_step_(*want, tau[:1], 1e-3)
+    row, v = q[0].clone(), qd[:1].clone()
+    m.rollout_step_(row, v, tau[:1], 1e-3)
+    assert torch.equal(row, want[0][0]) and torch.equal(v, want[1])
+    with pytest.raises(Exception):
+        m.rollout_step_(q[0].clone(), qd.clone(), tau, 1e-3)  # one environment against five
