@@ -136,8 +136,7 @@ int sapamd_get_chain_shape(const sapamd_model *m, int64_t B, int32_t *G, int32_t
  * kinematics of trees that are not short chains, and this model's segment of
  * a heterogeneous launch): 8, 16 or 32, at least the joint count; 0 (default) =
  * one per joint, environments back to back in a wavefront (the autotuner's
- * setting; no reference counterpart). With 0 set, get returns the smallest
- * group that holds the joints. */
+ * setting; no reference counterpart). get returns what was set. */
 int sapamd_set_tree_group(sapamd_model *m, int32_t G);
 int sapamd_get_tree_group(const sapamd_model *m, int32_t *G);
 /* Schedule of the lanes-per-joint CLIK launches, library-wide so that a

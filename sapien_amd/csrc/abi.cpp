@@ -150,10 +150,9 @@ struct sapamd_model {
   // Rollouts under the lanes-per-joint dynamics: one launch for all steps
   // (default), or one launch per step (the path graph-captured step loops use).
   bool per_step_rollouts = false;
-  // Lanes per environment of the lanes-per-joint tree kernels (0 = the
-  // smallest of 8, 16, 32 that holds the joints; the autotuner may pick more).
+  // Lanes per environment of the lanes-per-joint tree kernels: 8, 16 or 32, or
+  // 0 = one per joint, environments back to back.
   int tree_G = 0;
-  int tree_lanes() const { return tree_G ? tree_G : tree_group(host->njoints()); }
   // Lanes-per-joint forward dynamics: the factorization of M per root subtree
   // (M is block diagonal over them) when that shortens it; rows = its size.
   DynFactorPlan factor_plan() const {
@@ -895,7 +894,7 @@ int sapamd_set_tree_group(sapamd_model *m, int32_t G) {
 int sapamd_get_tree_group(const sapamd_model *m, int32_t *G) {
   return guarded([&] {
     if (!m || !G) throw std::invalid_argument("null argument");
-    *G = m->tree_lanes();
+    *G = m->tree_G;
   });
 }
 

@@ -159,6 +159,7 @@ def set_tree_group(model, G):
 
 
 def get_tree_group(model):
+    """The setting in effect (0: one lane per joint), so that it can be put back."""
     from .native import check, handle, lib
 
     g = ctypes.c_int32()

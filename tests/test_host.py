@@ -167,3 +167,17 @@ def test_philox_known_answers():
              (0xd16cfe09, 0x94fdcceb, 0x5001e420, 0x24126ea1))]
     for c, k, ref in kats:
         assert tuple(int(x) for x in philox4x32_10(*c, *k)) == ref
+
+
+@pytest.mark.parametrize("name", S.ROBOTS)
+def test_tree_group_setting_can_be_saved_and_put_back(name):
+    from sapien_amd import tune
+
+    rob = S.robot(name)
+    m = sa.PinocchioModel(rob.urdf, [0.0, 0.0, -9.81])
+    assert tune.get_tree_group(m) == 0  # the default: one lane per joint
+    for G in tune.tree_groups(m):
+        tune.set_tree_group(m, G)
+        assert tune.get_tree_group(m) == G
+        tune.set_tree_group(m, tune.get_tree_group(m))
+        assert tune.get_tree_group(m) == G
