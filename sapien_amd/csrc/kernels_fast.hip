@@ -155,7 +155,7 @@ __global__ __launch_bounds__(256) void k_chain_fused(const ModelTable<float> *__
   float *const prow = poses + e * (lay.pose_env ? lay.pose_env : (int64_t)L * 7);
   float *const jrow = Jout + e * (int64_t)(6 * nv);
   float *const trow = tau + e * lay.tau;
-  const int pl = (int)lay.pose_link;
+  const int64_t pl = lay.pose_link;
   // staged outputs: this wavefront's environments e0 .. e0 + nlive - 1, this
   // lane's environment at slot le of the wavefront's LDS runs
   constexpr int EPW = 64 / G;

@@ -106,7 +106,7 @@ __device__ __forceinline__ void tree_body(const ModelTable<float> *M, const Mode
   const int u = J.vuser;
   constexpr bool NT = true;  // streaming output stores (see st())
   float *const prow = io.poses + row_at(env0, row, io.pose_env, L * 7);
-  const int pl = io.pose_link ? (int)io.pose_link : 7;
+  const int64_t pl = io.pose_link ? io.pose_link : 7;
 
   // Jacobian columns and link poses first: their stores drain while the
   // dynamics compute
