@@ -1079,7 +1079,7 @@ int sapamd_passive_force_batched(const sapamd_model *m, int64_t B, const float *
 }
 
 int sapamd_fk_batched(const sapamd_model *m, int64_t B, const float *q, float *poses, void *stream) {
-  need(poses, "poses");
+  if (!poses) { g_last_error = "poses must not be null"; return SAPAMD_INVALID_ARGUMENT; }
   return sapamd_fk_jac_rnea_batched(m, B, q, nullptr, nullptr, poses, nullptr, nullptr, stream);
 }
 

@@ -5,6 +5,9 @@ drop-in class reproduces the reference's argument handling and error types
 (pinocchio/pinocchio_model.cpp:33-36, 64-70, 99-140, 150-151)."""
 import ctypes
 import os
+import subprocess
+import sys
+import textwrap
 import xml.etree.ElementTree as ET
 
 import numpy as np
@@ -181,3 +184,25 @@ def test_tree_group_setting_can_be_saved_and_put_back(name):
         assert tune.get_tree_group(m) == G
         tune.set_tree_group(m, tune.get_tree_group(m))
         assert tune.get_tree_group(m) == G
+
+
+def test_null_outputs_come_back_as_errors():
+    """A missing output of the single-output entry points is an error code and
+    a message. In a child process: an exception that crossed the C ABI would
+    end it."""
+    script = textwrap.dedent("""
+        import ctypes
+        import sapien_amd as sa
+        from sapien_amd import native, synthetic as S
+        rob = S.chain7()
+        m = sa.PinocchioModel(rob.urdf, [0.0, 0.0, -9.81])
+        L, h = native.lib(), native.handle(m)
+        for name, inputs, what in (("sapamd_fk_batched", 1, "poses"), ("sapamd_jacobian_batched", 1, "J"),
+                                   ("sapamd_rnea_batched", 3, "tau")):
+            f = getattr(L, name)
+            f.argtypes, f.restype = [ctypes.c_void_p, ctypes.c_int64] + [ctypes.c_void_p] * (inputs + 2), ctypes.c_int
+            assert f(h, 4, *[None] * (inputs + 2)) == 1, name
+            assert L.sapamd_last_error().decode() == what + " must not be null"
+        """)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    subprocess.run([sys.executable, "-c", script], env=dict(os.environ, PYTHONPATH=root), check=True, timeout=120)
