@@ -63,10 +63,16 @@ class _PoseTorqueLoss(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gloss):
         (grads,) = ctx.saved_tensors
-        scaled = (grads * _as(gloss.detach(), torch.float32)[:, None]).unbind(0)
-        if len(scaled) == 1:  # no torque term: velocities and accelerations have no part in the loss
-            scaled = scaled + (None, None)
-        out = tuple(None if d is None or g is None else _as(g, d) for g, d in zip(scaled, ctx.dtypes))
+        s = _as(gloss.detach(), torch.float32)[:, None]
+        need = ctx.needs_input_grad[1:4]
+        if all(need) and len(grads) == 3:
+            # one product for all three; .data: tensors over it that are not views to autograd (a view
+            # made here would refuse changes in place). 208 us a training pass of 8192 9-joint arms, 228
+            # with three products.
+            parts = [g.data for g in (grads * s).unbind(0)]
+        else:  # a product, and its memory, for each gradient asked for
+            parts = [grads[k] * s if need[k] and k < len(grads) else None for k in range(3)]
+        out = tuple(None if g is None else _as(g, d) for g, d in zip(parts, ctx.dtypes))
         return (None,) + out + (None, None, None)
 
 
