@@ -539,8 +539,7 @@ struct sapamd_model {
     return {t64(), host->njoints(), L(), host->max_depth(), ++ticket, done_of(d_buf)};
   }
   // Wait for the per-call kernel's ticket (a kernel that cannot deliver it ends
-  // the wait through its stream), then copy n doubles at `off` to dst (dst =
-  // nullptr: the caller reads h_buf). Waiting for the stream instead adds the
+  // the wait through its stream), then copy n doubles at `off` to dst. Waiting for the stream instead adds the
   // end-of-kernel release and the completion signal, about 5 us a call. Every
   // per-call method ends here, so no kernel still writes the buffer when the
   // next call reads it.
@@ -553,7 +552,7 @@ struct sapamd_model {
         if (__atomic_load_n(done, __ATOMIC_ACQUIRE) != ticket) throw DeviceError("the call's kernel did not finish");
       }
     }
-    if (dst) std::memcpy(dst, h_buf + off, n * sizeof(double));
+    std::memcpy(dst, h_buf + off, n * sizeof(double));
   }
   // serial chain of <= 16 joints: the G x C chain kernels apply
   bool chain_kernel() const { return host->njoints() >= 1 && host->is_chain() && host->njoints() <= 16; }
@@ -922,6 +921,7 @@ void fused_launch(const sapamd_model *m, int64_t B, int flags, const float *q, c
                                S(stream), m->tree_G, ev0, ev1));
     }
   } else {
+    // by the variant's name: trees past 32 joints report thread-per-environment
     if (ev0 || ev1) throw std::runtime_error("kernel timing events need the lanes-per-joint kernels");
     if (m->wave_lanes()) {  // trees of 33 to 64 joints, a wavefront per environment
       HIP_OK(launch_tree_fused(m->t32(), m->host->njoints(), m->L(), m->host->max_depth(), B, flags, q, qd, qdd, o,

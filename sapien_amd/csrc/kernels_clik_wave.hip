@@ -1,9 +1,9 @@
 // One CLIK problem per wavefront in FP64: compute_inverse_kinematics
 // (pinocchio_model.cpp:228-300), one configuration per call. Lane k owns chain
-// joint k (chains of up to 64 joints) with its constants in registers; what
-// depends on the link's pose alone (the SE(3) log, the damped 6x6 solve, the best
-// iterate's bookkeeping) every lane computes for itself, so an iteration needs no
-// barrier. Per iteration:
+// joint k (chains of up to 64 joints), its state in registers and its rotation's
+// constants in LDS; what depends on the link's pose alone (the SE(3) log, the
+// damped 6x6 solve, the best iterate's bookkeeping) every lane computes for
+// itself, so an iteration needs no barrier. Per iteration:
 //   FK      a prefix product of the joints' transforms over the lanes (DPP row
 //           shifts for chains of up to 16 joints, ds_bpermute past that), the
 //           link joint's pose read from its lane into scalars
@@ -14,7 +14,7 @@
 // Bound: latency, one wavefront's chain of about 1,100 instructions an
 // iteration. An arm of 7 joints and two fingers, about 75 iterations a call: 400 us
 // with one block whose thread 0 composed the chain and solved (six barriers an
-// iteration), 190 us here (2.5 us an iteration). The joints' constants stay in
+// iteration), 190 us here (2.5 us an iteration). The rotations' constants stay in
 // LDS: in registers the two-finger arm takes 183 us, but 12 joints 200 us instead
 // of 193 and 40 joints 341 us instead of 318 (the kernel then needs more than
 // the 256 registers an instruction can name).
@@ -100,7 +100,7 @@ __device__ __forceinline__ S6<double> log_blocks(const double *R, Vd p, double *
   }
   double al, be, db;
   if (t < 0.5) {
-    log_coeffs_dev(t, st, c, al, be, db);
+    log_series(t, al, be, db);
   } else {
     const double r = reciprocal(t), u = reciprocal(1.0 - c), r2 = r * r, hsu = 0.5 * st * u;
     al = t * hsu;

@@ -1,4 +1,4 @@
-// SE(3) helpers of the CLIK kernels (device, templated on float/double):
+// SE(3) helpers of the CLIK kernels (device; the batched kernels' log in FP32):
 // body-frame images of motion vectors, the SE(3) log and its Jacobian, and the
 // damped 6x6 solve, as used by compute_inverse_kinematics
 // (pinocchio_model.cpp:228-300).
@@ -37,8 +37,6 @@ __device__ __forceinline__ float rn_div_by(float a, float b) {  // b a constant
   const float r = 1.f / b, q = a * r;
   return fmaf(fmaf(-q, b, a), r, q);
 }
-__device__ __forceinline__ double rn_rcp(double x) { return 1.0 / x; }
-__device__ __forceinline__ double rn_div(double a, double b) { return a / b; }
 __device__ __forceinline__ double rn_div_by(double a, double b) { return a / b; }
 
 // Rotation log in the form Pinocchio 2.6 evaluates it (the reference's
@@ -50,54 +48,52 @@ __device__ __forceinline__ double rn_div_by(double a, double b) { return a / b; 
 // the signs of the skew part. For a rotation any correct log agrees; this
 // form also gives the reference's error vector when R is not orthonormal (a
 // target built from a quaternion that is not unit length).
-// s, c: sin and cos of the angle, for the coefficients as well (FP32).
-template <class T> __device__ __forceinline__ V3<T> log3_dev(const T *R, T &theta, T &s, T &c) {
-  const T PI = T(3.14159265358979323846);
-  const T tr = R[0] + R[4] + R[8];
-  theta = tr >= T(3) ? T(0) : tr <= T(-1) ? PI : acos((tr - T(1)) * T(0.5));
-  if constexpr (sizeof(T) == 4) sincosf(theta, &s, &c);
-  const V3<T> ax = {T(0.5) * (R[7] - R[5]), T(0.5) * (R[2] - R[6]), T(0.5) * (R[3] - R[1])};
-  if (theta < PI - T(1e-2)) {
-    constexpr bool fp64 = sizeof(T) == 8;
-    if constexpr (fp64) s = sin(theta);
-    const T k = theta > (fp64 ? T(1.220703125e-4) : T(1e-3)) ? rn_div(theta, s)
-                : fp64 ? T(1) : T(1) + theta * theta / T(6);
+// s, c: sin and cos of the angle, for the coefficients as well. FP32; the
+// per-call kernel has its own FP64 form.
+__device__ __forceinline__ V3<float> log3_dev(const float *R, float &theta, float &s, float &c) {
+  const float PI = 3.14159265358979323846f;
+  const float tr = R[0] + R[4] + R[8];
+  theta = tr >= 3.f ? 0.f : tr <= -1.f ? PI : acos((tr - 1.f) * 0.5f);
+  sincosf(theta, &s, &c);
+  const V3<float> ax = {0.5f * (R[7] - R[5]), 0.5f * (R[2] - R[6]), 0.5f * (R[3] - R[1])};
+  if (theta < PI - 1e-2f) {
+    const float k = theta > 1e-3f ? rn_div(theta, s) : 1.f + theta * theta / 6.f;
     return k * ax;
   }
-  if constexpr (sizeof(T) == 8) c = cos(theta);
-  const T b = rn_div(theta * theta, T(1) - c);
-  const T x0 = (R[0] - c) * b, x1 = (R[4] - c) * b, x2 = (R[8] - c) * b;
-  return {(R[7] > R[5] ? T(1) : T(-1)) * (x0 > T(0) ? sqrt(x0) : T(0)),
-          (R[2] > R[6] ? T(1) : T(-1)) * (x1 > T(0) ? sqrt(x1) : T(0)),
-          (R[3] > R[1] ? T(1) : T(-1)) * (x2 > T(0) ? sqrt(x2) : T(0))};
+  const float b = rn_div(theta * theta, 1.f - c);
+  const float x0 = (R[0] - c) * b, x1 = (R[4] - c) * b, x2 = (R[8] - c) * b;
+  return {(R[7] > R[5] ? 1.f : -1.f) * (x0 > 0.f ? sqrt(x0) : 0.f), (R[2] > R[6] ? 1.f : -1.f) * (x1 > 0.f ? sqrt(x1) : 0.f),
+          (R[3] > R[1] ? 1.f : -1.f) * (x2 > 0.f ? sqrt(x2) : 0.f)};
 }
 
-// alpha = (t/2) cot(t/2), beta = (1 - alpha) / t^2, dbeta = beta'(t) / t; series
-// below 0.5. st, ct: log3_dev's sin t and cos t (FP32).
-template <class T> __device__ __forceinline__ void log_coeffs_dev(T t, T st, T ct, T &alpha, T &beta, T &dbeta) {
-  T t2 = t * t;
-  if (t < T(0.5)) {
-    alpha = T(1) - t2 * (T(1) / T(12) + t2 * (T(1) / T(720) + t2 * (T(1) / T(30240) + rn_div_by(t2, T(1209600)))));
-    beta = T(1) / T(12) +
-           t2 * (T(1) / T(720) + t2 * (T(1) / T(30240) + t2 * (T(1) / T(1209600) + rn_div_by(t2, T(47900160)))));
-    dbeta = T(1) / T(360) + t2 * (T(1) / T(7560) + t2 * (T(1) / T(201600) + rn_div_by(t2, T(5987520))));
+// alpha = (t/2) cot(t/2), beta = (1 - alpha) / t^2, dbeta = beta'(t) / t: the
+// series, for t below 0.5.
+template <class T> __device__ __forceinline__ void log_series(T t, T &alpha, T &beta, T &dbeta) {
+  const T t2 = t * t;
+  alpha = T(1) - t2 * (T(1) / T(12) + t2 * (T(1) / T(720) + t2 * (T(1) / T(30240) + rn_div_by(t2, T(1209600)))));
+  beta = T(1) / T(12) +
+         t2 * (T(1) / T(720) + t2 * (T(1) / T(30240) + t2 * (T(1) / T(1209600) + rn_div_by(t2, T(47900160)))));
+  dbeta = T(1) / T(360) + t2 * (T(1) / T(7560) + t2 * (T(1) / T(201600) + rn_div_by(t2, T(5987520))));
+}
+// st, ct: log3_dev's sin t and cos t.
+__device__ __forceinline__ void log_coeffs_dev(float t, float st, float ct, float &alpha, float &beta, float &dbeta) {
+  if (t < 0.5f) {
+    log_series(t, alpha, beta, dbeta);
   } else {
-    if constexpr (sizeof(T) == 8) sincos(t, &st, &ct);
     // two reciprocals (1/t, 1/(1 - cos t)) instead of one division per term
-    const T r = rn_rcp(t), u = rn_rcp(T(1) - ct), r2 = r * r, hsu = T(0.5) * st * u;
+    const float r = rn_rcp(t), u = rn_rcp(1.f - ct), r2 = r * r, hsu = 0.5f * st * u;
     alpha = t * hsu;
     beta = r2 - r * hsu;
-    dbeta = T(-2) * r2 * r2 + (T(1) + st * r) * (T(0.5) * u) * r2;
+    dbeta = -2.f * r2 * r2 + (1.f + st * r) * (0.5f * u) * r2;
   }
 }
 
-template <class T>
-__device__ __forceinline__ S6<T> log6_dev(const T *R, V3<T> p) {
-  T t, st, ct;
-  V3<T> w = log3_dev(R, t, st, ct);
-  T al, be, db;
+__device__ __forceinline__ S6<float> log6_dev(const float *R, V3<float> p) {
+  float t, st, ct;
+  V3<float> w = log3_dev(R, t, st, ct);
+  float al, be, db;
   log_coeffs_dev(t, st, ct, al, be, db);
-  return {al * p - T(0.5) * cross(w, p) + (be * dot(w, p)) * w, w};
+  return {al * p - 0.5f * cross(w, p) + (be * dot(w, p)) * w, w};
 }
 
 // Jlog6 (6x6 row-major): [[A, C A], [0, A]], A = alpha I + beta w w^T + [w]x / 2,
@@ -118,25 +114,24 @@ __device__ __forceinline__ void jlog6_blocks(V3<T> w, T t, T al, T be, T db, V3<
   C[1] -= T(0.5) * p.z; C[2] += T(0.5) * p.y; C[5] -= T(0.5) * p.x;
   C[3] += T(0.5) * p.z; C[6] -= T(0.5) * p.y; C[7] += T(0.5) * p.x;
 }
-template <class T>
-__device__ __forceinline__ void jlog6_core(V3<T> w, T t, T al, T be, T db, V3<T> p, T *Jl) {
-  T A[9], C[9];
+__device__ __forceinline__ void jlog6_core(V3<float> w, float t, float al, float be, float db, V3<float> p, float *Jl) {
+  float A[9], C[9];
   jlog6_blocks(w, t, al, be, db, p, A, C);
-  T CA[9];
+  float CA[9];
   mm(C, A, CA);
   for (int i = 0; i < 3; ++i)
     for (int j = 0; j < 3; ++j) {
       Jl[i * 6 + j] = A[3 * i + j];
       Jl[i * 6 + 3 + j] = CA[3 * i + j];
-      Jl[(3 + i) * 6 + j] = T(0);
+      Jl[(3 + i) * 6 + j] = 0.f;
       Jl[(3 + i) * 6 + 3 + j] = A[3 * i + j];
     }
 }
 
-template <class T> __device__ __forceinline__ void jlog6_dev(const T *R, V3<T> p, T *Jl) {
-  T t, st, ct;
-  V3<T> w = log3_dev(R, t, st, ct);
-  T al, be, db;
+__device__ __forceinline__ void jlog6_dev(const float *R, V3<float> p, float *Jl) {
+  float t, st, ct;
+  V3<float> w = log3_dev(R, t, st, ct);
+  float al, be, db;
   log_coeffs_dev(t, st, ct, al, be, db);
   jlog6_core(w, t, al, be, db, p, Jl);
 }
@@ -146,30 +141,29 @@ template <class T> __device__ __forceinline__ void jlog6_dev(const T *R, V3<T> p
 // the coefficients are the same; in the branch near pi the signs come from the
 // skew part, which also flips, unless two of its entries tie exactly), so this
 // equals log6_dev(R, p) and jlog6_dev(R^T, -R^T p) bit for bit.
-template <class T> __device__ __forceinline__ S6<T> log6_jlog6_inv(const T *R, V3<T> p, T *Jl) {
-  T t, st, ct;
-  V3<T> w = log3_dev(R, t, st, ct);
-  T al, be, db;
+__device__ __forceinline__ S6<float> log6_jlog6_inv(const float *R, V3<float> p, float *Jl) {
+  float t, st, ct;
+  V3<float> w = log3_dev(R, t, st, ct);
+  float al, be, db;
   log_coeffs_dev(t, st, ct, al, be, db);
-  jlog6_core(T(-1) * w, t, al, be, db, T(-1) * mtv(R, p), Jl);
-  return {al * p - T(0.5) * cross(w, p) + (be * dot(w, p)) * w, w};
+  jlog6_core(-1.f * w, t, al, be, db, -1.f * mtv(R, p), Jl);
+  return {al * p - 0.5f * cross(w, p) + (be * dot(w, p)) * w, w};
 }
 // The same with Jlog6(M^-1) as its blocks A, C: Jlog6 v = [A v_l + C (A v_a); A v_a]
 // costs 27 products per column instead of 36, and C A is never formed.
-template <class T> __device__ __forceinline__ S6<T> log6_jlog6_inv_blocks(const T *R, V3<T> p, T *A, T *C) {
-  T t, st, ct;
-  V3<T> w = log3_dev(R, t, st, ct);
-  T al, be, db;
+__device__ __forceinline__ S6<float> log6_jlog6_inv_blocks(const float *R, V3<float> p, float *A, float *C) {
+  float t, st, ct;
+  V3<float> w = log3_dev(R, t, st, ct);
+  float al, be, db;
   log_coeffs_dev(t, st, ct, al, be, db);
-  jlog6_blocks(T(-1) * w, t, al, be, db, T(-1) * mtv(R, p), A, C);
-  return {al * p - T(0.5) * cross(w, p) + (be * dot(w, p)) * w, w};
+  jlog6_blocks(-1.f * w, t, al, be, db, -1.f * mtv(R, p), A, C);
+  return {al * p - 0.5f * cross(w, p) + (be * dot(w, p)) * w, w};
 }
 
 // 1 / d as the compiler's FP64 division computes it (hardware reciprocal, two
 // Newton steps, one residual correction, the fix-up of zeros, infinities and
 // NaN) without that division's scaling, which only matters for pivots beyond
 // 2^+-1000: the same bits in 8 instructions instead of 12, in a serial chain.
-__device__ __forceinline__ float pivot_rcp(float d) { return 1.f / d; }
 __device__ __forceinline__ double pivot_rcp(double d) {
   double r = __builtin_amdgcn_rcp(d);
 #pragma unroll
