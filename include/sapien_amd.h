@@ -155,8 +155,8 @@ int sapamd_fk_jac_rnea_batched(const sapamd_model *m, int64_t B, const float *q,
 /* The same launch with the kernel's own start and stop recorded into two
  * caller-created hipEvent_t (hipExtLaunchKernel), so hipEventElapsedTime gives
  * the kernel's execution time without the dispatch gaps around it: kernel
- * timing without a profiler (lanes-per-joint kernels only; not for graph
- * capture). No reference counterpart. */
+ * timing without a profiler (models whose variant is lanes-per-joint, so trees
+ * of up to 32 joints; not for graph capture). No reference counterpart. */
 int sapamd_fk_jac_rnea_batched_timed(const sapamd_model *m, int64_t B, const float *q, const float *qd,
                                      const float *qdd, float *poses, float *J, float *tau, void *start_event,
                                      void *stop_event, void *stream);

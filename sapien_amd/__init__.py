@@ -4,7 +4,8 @@ Drop-in for SAPIEN's ``PinocchioModel`` (python/py_package/wrapper/pinocchio_mod
 pinocchio/pinocchio_model.cpp): the same class, method and argument names, with
 every computation running in hand-written HIP kernels for gfx950 behind the C
 ABI of ``include/sapien_amd.h``. Batched ``*_batched`` methods take (B, dof)
-tensors through DLPack.
+tensors: torch tensors on the model's GPU in place, anything else through
+torch's conversions or DLPack.
 
 The native extension is required: importing this package without it raises.
 """

@@ -1,7 +1,7 @@
 // The per-call methods (one configuration, FP64, the reference's use): one
 // wavefront per call, lane j owning joint j of the depth-first order (trees of up
-// to 64 joints), inputs read from and results written to the model's pinned
-// per-call buffer.
+// to 64 joints), inputs handed over as kernel arguments and results written to
+// the model's pinned per-call buffer.
 //   X, v, a      root to joint: pointer jumping with ds_bpermute, log2(depth) rounds
 //   F, Ic, ABA   leaves to root: level by level through LDS, a joint adding its
 //                children's values (their lanes are j + 1 and then each

@@ -1,7 +1,7 @@
 // Lanes-per-joint Coriolis matrices and per-link Jacobians (FP32) for trees of
-// up to 64 joints: one environment per group of G lanes (G = 8, 16, 32, or a
-// whole wavefront of 64), lane j owning joint j of the depth-first order, with
-// the tree scans of tree.h.
+// up to 64 joints, lane j owning joint j of the depth-first order, with the tree
+// scans of tree.h: the Coriolis kernel packs environments back to back, a lane
+// per joint, the Jacobian kernel gives each a group of 8, 16, 32 or 64 lanes.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -65,11 +65,12 @@ __device__ __forceinline__ int64_t row_at(int64_t env0, int row, int64_t ld, int
 // the staged table and, at 4 cycles a SIMD, 780 VALU instructions have to fit. So
 // what pays is a wavefront's exchanges serving more environments: 7 of 9 joints
 // instead of 4 in groups of 16 lanes, and only the pointer-jumping rounds that
-// the deepest joint needs. 524287 environments of that tree: 236 us in 16-lane
-// groups, 133 us packed, 126 with the subtree sums' first two rounds as
+// the deepest joint needs. 524287 environments of that tree, a call: 212 us in
+// 16-lane groups, 135 us packed, 126 with the subtree sums' first two rounds as
 // wavefront shifts (337 MB, 72 us at a copy's rate): the LDS pipe is busy for
 // 110 us of it with 131 exchanges a wavefront, the vector units for 93. Poses
-// and Jacobians staged through LDS for whole-sector stores: 155 us (packed: 138).
+// and Jacobians staged through LDS for whole-sector stores: 155 us (packed then:
+// 138).
 template <int G, bool SPARE>
 __device__ __forceinline__ void tree_body(const ModelTable<float> *M, const ModelTable<float> *__restrict__ Mg,
                                           int64_t B, int64_t wave, int flags, const TreeIO &io, float *lds) {
@@ -510,6 +511,17 @@ __global__ __launch_bounds__(256) void k_hetero(HeteroArgs args, int flags, int 
 
 int tree_group(int nj) { return nj < 1 ? 0 : nj <= 8 ? 8 : nj <= 16 ? 16 : nj <= 32 ? 32 : 0; }
 
+// lanes = 0, the default, is back to back at every batch. Against groups of 8, 16
+// or 32 lanes it gains where more environments fit a wavefront and the batch
+// fills the chip, and loses up to 8 % below that, where fewer wavefronts have
+// more to do each. Fused kinematics, us a launch, packed / smallest group that
+// holds the joints (environments a wavefront):
+//   batch             4096        8192         16384        65536       262144
+//   9 joints (7/4)    5.8/5.5    6.8/6.4      8.4/9.0    24.0/24.9   70.9/93.0
+//   18 joints (3/2)   7.6/7.3    9.5/10.9    15.3/18.3   44.7/61.1    168/235
+//   30 joints (2/2)   8.1/7.9   12.1/11.5    19.4/18.9   65.1/64.1    255/247
+// The mixed launch of four trees x 8192: 12.9 packed, 12.3 with 8 / 16 / packed /
+// 32, which the autotuner finds.
 TreePacking tree_packing(int nj, int nlinks, int max_depth, int lanes) {
   TreePacking p;
   p.nj = nj;

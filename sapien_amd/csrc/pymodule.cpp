@@ -473,7 +473,7 @@ class PyModel {
     return py::make_tuple(lo, hi);
   }
 
-  // ---------------------------------------------------------------- batched (DLPack, FP32)
+  // ---------------------------------------------------------------- batched (FP32)
   py::object fk_jac_rnea_batched(py::object q, py::object qd, py::object qdd, bool poses, bool jac, bool rnea,
                                  py::object stream) {
     StreamScope scope_(stream, info().device);
@@ -689,7 +689,7 @@ class PyModel {
     return py::make_tuple(Q, Sx, E, I, solved);
   }
 
-  // ---------------------------------------------------------------- adjoints (DLPack, FP32)
+  // ---------------------------------------------------------------- adjoints (FP32)
   py::tuple kin_vjp_batched(py::object q, py::object qd, py::object qdd, py::object gposes, py::object gtau,
                             py::object stream) {
     StreamScope scope_(stream, info().device);
@@ -774,7 +774,7 @@ class PyModel {
     return py::make_tuple(loss, tau, dq, dqd, dqdd);
   }
 
-  // ---------------------------------------------------------------- rollouts (DLPack, FP32)
+  // ---------------------------------------------------------------- rollouts (FP32)
   // (T, K) of a (B, T, nv) torque tensor and a checkpoint interval
   static int32_t ckpt_count(int64_t T, int64_t K) { return (int32_t)((T + K - 1) / K); }
   py::tuple rollout_batched(py::object q0, py::object qd0, py::object tau, double dt, int64_t K, py::object stream) {
@@ -1306,7 +1306,7 @@ PYBIND11_MODULE(_pinocchio, m) {
       .def_property_readonly("nlinks", [](const PyModel &s) { return s.info().nlinks; })
       .def_property_readonly("is_chain", [](const PyModel &s) { return bool(s.info().chain); })
       .def_property_readonly("max_depth", [](const PyModel &s) { return s.info().max_depth; })
-      // batched FP32 methods over (B, dof) tensors (DLPack, kDLROCM)
+      // batched FP32 methods over (B, dof) tensors
       .def("compute_forward_kinematics_batched", &PyModel::fk_batched, py::arg("qpos"), py::arg("stream") = py::none(),
            "Link poses (B, L, 7) = p xyz | q wxyz for a (B, nv) batch.")
       .def("compute_full_jacobian_batched", &PyModel::jac_batched, py::arg("qpos"), py::arg("stream") = py::none(),
