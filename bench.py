@@ -177,8 +177,8 @@ def traffic_of(traffic, shape, variant):
     """The figures of the kernel the timed run used, from measure_traffic."""
     if not traffic:
         return None
-    key = f"k_chain_fused<{shape[0]}, {shape[1]}>" if shape else ("k_kinematics" if variant != "lanes_per_joint"
-                                                                  else "k_tree_fused")
+    key = f"k_chain_fused<{shape[0]}, {shape[1]}, " if shape else ("k_kinematics" if variant != "lanes_per_joint"
+                                                                   else "k_tree_fused")
     for name, v in traffic.items():
         if key in name and "FETCH_SIZE" in v and "WRITE_SIZE" in v:
             return v

@@ -49,7 +49,9 @@ struct Layout {
   int32_t staged, per_wave;
 };
 
-template <int G, int C>
+// STAGE: the kernel can stage its outputs (lay.staged); without it, a small
+// launch is spared the code (launch_chain_fused).
+template <int G, int C, bool STAGE>
 __global__ __launch_bounds__(256) void k_chain_fused(const ModelTable<float> *__restrict__ Mg, int64_t B, int flags,
                                                      const float *__restrict__ q, const float *__restrict__ qd,
                                                      const float *__restrict__ qdd, float *__restrict__ poses,
@@ -159,7 +161,7 @@ __global__ __launch_bounds__(256) void k_chain_fused(const ModelTable<float> *__
   // staged outputs: this wavefront's environments e0 .. e0 + nlive - 1, this
   // lane's environment at slot le of the wavefront's LDS runs
   constexpr int EPW = 64 / G;
-  const bool staged = G >= 4 && lay.staged;
+  const bool staged = STAGE && lay.staged;
   const int le = IL ? (((lane >> 4) << 1) | (lane & 1)) : lane / G;
   const int64_t e0 = (blockIdx.x * (int64_t)blockDim.x + (threadIdx.x & ~63)) / G;
   const int nlive = (int)(B - e0 < EPW ? (B - e0 > 0 ? B - e0 : 0) : EPW);
@@ -315,12 +317,15 @@ void launch_gc(const ModelTable<float> *tab, int64_t B, int flags, const float *
   const int64_t envs_per_block = 256 / G;
   dim3 grid((unsigned)((B + envs_per_block - 1) / envs_per_block));
   const unsigned lds = lay.staged ? 4u * (unsigned)lay.per_wave * (unsigned)sizeof(float) : 0u;  // 4 wavefronts
+  auto kernel = k_chain_fused<G, C, (G >= 4)>;
+  if constexpr (G == 4)
+    if (!lay.staged) kernel = k_chain_fused<G, C, false>;
   if (ev0 || ev1)  // the kernel's own start and stop recorded into the caller's events
-    hipExtLaunchKernelGGL((k_chain_fused<G, C>), grid, dim3(256), lds, s, ev0, ev1, 0, tab, B, flags, q, qd, qdd,
-                          out.poses, out.jfull, out.tau, lay);
+    hipExtLaunchKernelGGL(kernel, grid, dim3(256), lds, s, ev0, ev1, 0, tab, B, flags, q, qd, qdd, out.poses,
+                          out.jfull, out.tau, lay);
   else
-    hipLaunchKernelGGL((k_chain_fused<G, C>), grid, dim3(256), lds, s, tab, B, flags, q, qd, qdd, out.poses,
-                       out.jfull, out.tau, lay);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), lds, s, tab, B, flags, q, qd, qdd, out.poses, out.jfull, out.tau,
+                       lay);
 }
 
 }  // namespace
@@ -361,10 +366,14 @@ hipError_t launch_chain_fused(const ModelTable<float> *tab, int nj, int64_t B, i
   lay.pose_env = out.pose_env;  // 0: L * 7, resolved in the kernel from the table
   // staged outputs for 4 and more lanes per environment over contiguous outputs
   // (the pose run assumes at most one link per joint plus the root, checked in the
-  // kernel). 4 lanes x 2 joints, 7-joint chain: 524288 environments 95 -> 65 us,
-  // 65536 16.5 -> 12.0 us, 16384 8.5 -> 8.1 us. With 1 or 2 lanes a wavefront's
-  // runs (27 KB and more) leave no room for a second block on the CU.
-  lay.staged = G >= 4 && out.pose_env == 0 && lay.pose_link == 7 && lay.tau == nv ? 1 : 0;
+  // kernel). With 1 or 2 lanes a wavefront's runs (27 KB and more) leave no room
+  // for a second block on the CU. With 4 lanes the detour pays once the stores
+  // bound the launch: 7-joint chain, rows / staged us: 5.8 / 6.2 at 4096
+  // environments, 6.8 / 6.5 at 12288, 10.7 / 7.9 at 32768, 49 / 35 at 262144; poses
+  // alone of a 3-joint chain 6.5 / 6.7 at 65536, torques alone 24.5 / 25.6 at 262144.
+  const bool bulk = (flags & KF_JFULL) ? nj >= 2 : (flags & KF_POSES) && nj >= 4;
+  const bool pays = G >= 8 || (G == 4 && bulk && B * nj >= 98304);
+  lay.staged = pays && out.pose_env == 0 && lay.pose_link == 7 && lay.tau == nv ? 1 : 0;
   lay.per_wave = (64 / G) * (6 * nv + 7 * (nj + 1) + nv);  // a multiple of 4: the runs stay 16-byte aligned
   // bits 2, 4, 8: the J, pose and tau runs start 16-byte aligned (each
   // wavefront's run starts a multiple of 16 bytes after the array's start)
