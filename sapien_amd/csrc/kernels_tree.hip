@@ -105,7 +105,12 @@ __device__ __forceinline__ void tree_body(const ModelTable<float> *M, const Mode
   T.prefix(X);
   const S6<float> col = valid ? jcol(J, X.R, X.p) : zero6<float>();
   const int u = J.vuser;
-  constexpr bool NT = true;  // streaming output stores (see st())
+  // Streaming output stores (see st()), except up to 8 joints: their rows are
+  // shorter than a 64-byte sector, and of plain stores the L2 cache merges the
+  // pieces. 5-joint tree x 262144: 95 us streaming, 31 us so (42 with one
+  // environment per 8 lanes, streaming); 8 joints x 65536 20.1 and 15.7, x 16384,
+  // which the cache holds, 6.7 and 7.0.
+  constexpr bool NT = G > 8;
   float *const prow = io.poses + row_at(env0, row, io.pose_env, L * 7);
   const int64_t pl = io.pose_link ? io.pose_link : 7;
 
@@ -175,7 +180,7 @@ __device__ __forceinline__ void tree_body(const ModelTable<float> *M, const Mode
     } else {
       T.subtree(f);
     }
-    if (live && valid) st<NT>(dot6(col, f), io.tau + row_at(env0, row, io.ld_tau, nv) + u);
+    if (live && valid) st<true>(dot6(col, f), io.tau + row_at(env0, row, io.ld_tau, nv) + u);
   }
   if (do_crba) {
     if (!dyn) T.template subtree<10>(y);
