@@ -45,6 +45,7 @@ struct TreeIO {
 // for one environment of 64 joints).
 constexpr int tree_waves(int width) { return width > 32 ? 2 : 4; }
 int tree_wave_floats(const TreePacking &p) {
+  if (p.dense) return 64 * 12;
   return AncestorRows<1>::kFloats + ((p.per_wave * p.nj * p.nj + 3) & ~3);
 }
 
@@ -190,6 +191,33 @@ __device__ __forceinline__ void tree_body(const ModelTable<float> *M, const Mode
 #pragma unroll
     for (int i = 0; i < 6; ++i) Yc.I[i] = y[4 + i];
     const S6<float> Fj = apply(Yc, col);
+    if (io.pack.dense) {
+      // Deep trees: M is nearly full. Every lane publishes its column and force,
+      // lane j reads those of all joints of its environment (one address across
+      // it at a time) and stores row u of M, entry (i, u) for (u, i): at each i an
+      // environment writes one contiguous row. A 32-joint chain x 65536: 109 us so,
+      // 160 by the walk below; 30 joints 100 and 116; 16 joints 39 and 47.
+      float4 *const cf = reinterpret_cast<float4 *>(lds);
+      cf[T.lane * 3 + 0] = make_float4(col.l.x, col.l.y, col.l.z, col.a.x);
+      cf[T.lane * 3 + 1] = make_float4(col.a.y, col.a.z, Fj.l.x, Fj.l.y);
+      cf[T.lane * 3 + 2] = make_float4(Fj.l.z, Fj.a.x, Fj.a.y, Fj.a.z);
+      wave_sync();
+      const bool out = live && valid;
+      const float4 *const ce = cf + (out ? T.base4 / 4 : 0) * 3;
+      float *const Mcol = io.M + env0 * nv * nv + __umul24(row, nv * nv) + u;
+#pragma unroll 4
+      for (int i = 0; i < nj; ++i) {
+        const float4 r0 = ce[i * 3 + 0], r1 = ce[i * 3 + 1], r2 = ce[i * 3 + 2];
+        const S6<float> ci = {{r0.x, r0.y, r0.z}, {r0.w, r1.x, r1.y}};
+        const S6<float> Fi = {{r1.z, r1.w, r2.x}, {r2.y, r2.z, r2.w}};
+        // joint i's subtree size and user dof: on lane i, the first environment's
+        const int sub_i = __builtin_amdgcn_readlane(T.size, i), ui = __builtin_amdgcn_readlane(u, i);
+        const float dij = dot6(ci, Fj), dji = dot6(col, Fi);
+        const bool i_anc_j = i <= g && g < i + sub_i, j_anc_i = g < i && i < g + T.size;
+        if (out) Mcol[__umul24(ui, nv)] = i_anc_j ? dij : j_anc_i ? dji : 0.f;
+      }
+      return;
+    }
     // M is nonzero between a joint and its ancestors: every lane publishes its
     // column, lane j walks its ancestors i and puts col_i . F_j at (i, j) and
     // (j, i) of the wavefront's LDS tile, whose environments then leave as one
@@ -534,6 +562,10 @@ TreePacking tree_packing(int nj, int nlinks, int max_depth, int lanes) {
   p.max_depth = max_depth;
   p.rounds = 0;
   while ((1 << p.rounds) < max_depth) ++p.rounds;
+  // M row by row where a joint has most others as ancestors; past 32 joints the
+  // walk over the ancestors is the faster one at small batches (64 joints x 64:
+  // 13.7 us, 15.5 row by row).
+  p.dense = nj <= 32 && 4 * max_depth > 3 * nj;
   p.stride = lanes ? lanes : nj;
   p.per_wave = 64 / p.stride;
   p.magic = 65536 / p.stride + 1;

@@ -38,6 +38,7 @@ struct TreePacking {
   int32_t stride, per_wave, magic, spare, width;
   int32_t nj, nlinks;
   int32_t max_depth, rounds;  // longest root-to-leaf joint chain; 2^rounds >= max_depth
+  int32_t dense;  // M: rows over all joints instead of a walk over the ancestors
 };
 // Environments of nj joints at `lanes` lanes each (0 = nj, back to back).
 TreePacking tree_packing(int nj, int nlinks, int max_depth, int lanes);
