@@ -544,17 +544,16 @@ __global__ __launch_bounds__(256) void k_hetero(HeteroArgs args, int flags, int 
 
 int tree_group(int nj) { return nj < 1 ? 0 : nj <= 8 ? 8 : nj <= 16 ? 16 : nj <= 32 ? 32 : 0; }
 
-// lanes = 0, the default, is back to back at every batch. Against groups of 8, 16
-// or 32 lanes it gains where more environments fit a wavefront and the batch
-// fills the chip, and loses up to 8 % below that, where fewer wavefronts have
-// more to do each. Fused kinematics, us a launch, packed / smallest group that
-// holds the joints (environments a wavefront):
-//   batch             4096        8192         16384        65536       262144
-//   9 joints (7/4)    5.8/5.5    6.8/6.4      8.4/9.0    24.0/24.9   70.9/93.0
-//   18 joints (3/2)   7.6/7.3    9.5/10.9    15.3/18.3   44.7/61.1    168/235
-//   30 joints (2/2)   8.1/7.9   12.1/11.5    19.4/18.9   65.1/64.1    255/247
-// The mixed launch of four trees x 8192: 12.9 packed, 12.3 with 8 / 16 / packed /
-// 32, which the autotuner finds.
+// lanes = 0, the default, is back to back at every batch. Fused kinematics, us a
+// launch, packed / smallest group that holds the joints (environments a
+// wavefront):
+//   batch             1024        4096        8192        16384       65536       262144
+//   9 joints (7/4)    5.5/5.2     5.8/5.5     6.5/6.3     8.4/8.7    26.6/25.6   69.5/94.7
+//   18 joints (3/2)   6.1/6.1     7.4/7.3     9.0/10.6   14.9/18.0   44.7/60.8    167/235
+//   30 joints (2/2)   6.4/6.3     7.7/7.6    11.1/10.9   19.1/18.7   64.9/64.2    251/246
+// Below about 8192 environments, where fewer wavefronts have more to do each, the
+// groups are up to 5 % faster; the mixed launch of four trees x 8192 takes 12.9
+// packed and 12.3 with 8 / 16 / packed / 32, which the autotuner finds.
 TreePacking tree_packing(int nj, int nlinks, int max_depth, int lanes) {
   TreePacking p;
   p.nj = nj;
