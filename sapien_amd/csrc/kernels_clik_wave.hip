@@ -12,9 +12,10 @@
 //   solve   L D L^T in every lane
 //
 // Bound: latency, one wavefront's chain of about 1,100 instructions an
-// iteration. An arm of 7 joints and two fingers, about 75 iterations a call: 400 us
+// iteration. An arm of 7 joints and two fingers, about 80 iterations a call: 400 us
 // with one block whose thread 0 composed the chain and solved (six barriers an
-// iteration), 190 us here (2.5 us an iteration). The rotations' constants stay in
+// iteration), 190 us here (2.25 us an iteration, 2.46 for 12 joints, 3.42 for 40,
+// over calls that run to the iteration limit). The rotations' constants stay in
 // LDS: in registers the two-finger arm takes 183 us, but 12 joints 200 us instead
 // of 193 and 40 joints 341 us instead of 318 (the kernel then needs more than
 // the 256 registers an instruction can name).

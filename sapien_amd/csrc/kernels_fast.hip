@@ -39,7 +39,7 @@ constexpr int kTableWords4 = (int)((kHeaderBytes + sizeof(JointRec<float>) * kMa
 
 // Row strides of the batched arrays, resolved on the host (elements).
 // staged: the outputs are contiguous (poses (B, L, 7), J (B, 6, nv), tau
-// (B, nv)) and an environment has at least 4 lanes: each wavefront's outputs,
+// (B, nv)) and staging them pays (launch_chain_fused): each wavefront's outputs,
 // whose environments are consecutive, go through per-wavefront LDS of
 // per_wave floats and leave as contiguous runs, every store instruction
 // writing 256 consecutive bytes (whole 64-byte sectors), instead of 28-byte
